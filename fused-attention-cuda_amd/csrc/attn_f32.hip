@@ -1,4 +1,4 @@
-// attn_f32.hip -- stage 3, fp32 compute: fp32 inputs on split fp16 operands, fp16 inputs on fp32 MFMA.
+// attn_f32.hip -- stage 3, fp32 compute: fp32 inputs on split bf16 operands, fp16 inputs on fp32 MFMA.
 #include "attn_kernel.h"
 #include "attn_split32.h"
 

@@ -1,7 +1,7 @@
 // attn_kernel.h -- the fp32-compute correctness rung of the fused SDPA forward (stage 3).
 //
 // Included by attn_f32.hip, which instantiates it for fp16 inputs, and by attn_split32.h, whose fp32
-// kernel falls back to it (Attn<float, ...>) on inputs outside fp16's range:
+// kernel falls back to it (Attn<float, ...>) on magnitudes that it does not split:
 //   fa_s3_fused<T>   (stage 3)  operands are held in LDS as fp32 and multiplied on
 //                               v_mfma_f32_32x32x2_f32, so no operand is rounded below fp32
 //                               (fp32 or fp16 I/O, ref:src/stage3_fused.cu:142-160). K/V tiles are
@@ -421,12 +421,20 @@ struct Attn {
     const float lt = halves_sum(ws.l);
     if (!wave_valid) return;
     const float inv = (lt > 0.f) ? 1.f / lt : 0.f;
-    Tio* orow = static_cast<Tio*>(a.o) + b * a.osb + h * a.osh + row * a.osn;
+    // With helper waves the lane again: kept over the walk it costs registers that the fp32 split kernel,
+    // which falls back to this one, does not have.
+    const int out_lane =
+        THREADS == 64 * WAVES
+            ? lane
+            : static_cast<int>(__builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u)));
+    const int out_g = out_lane >> 5;
+    const int out_row = r0 + (out_lane & 31);
+    Tio* orow = static_cast<Tio*>(a.o) + b * a.osb + h * a.osh + out_row * a.osn;
 #pragma unroll
     for (int db = 0; db < kDB; ++db) {
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
-        const int d = 32 * db + 8 * j + 4 * g;
+        const int d = 32 * db + 8 * j + 4 * out_g;
         const float x0 = ws.o[db][4 * j + 0] * inv, x1 = ws.o[db][4 * j + 1] * inv;
         const float x2 = ws.o[db][4 * j + 2] * inv, x3 = ws.o[db][4 * j + 3] * inv;
         if constexpr (__is_same(Tio, float)) {
@@ -437,8 +445,8 @@ struct Attn {
         }
       }
     }
-    if (g == 0) {
-      a.lse[(static_cast<size_t>(b) * a.H + h) * static_cast<size_t>(N) + row] =
+    if (out_g == 0) {
+      a.lse[(static_cast<size_t>(b) * a.H + h) * static_cast<size_t>(N) + out_row] =
           (lt > 0.f && ws.m != -__builtin_inff()) ? ws.m * a.scale + log2_hw(lt) * kLn2
                                                    : __builtin_inff();
     }
