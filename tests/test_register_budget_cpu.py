@@ -69,12 +69,21 @@ def test_every_kernel_is_spill_and_scratch_free(kernels):
 
 
 def test_every_kernel_was_reported(kernels):
-    families = {"fa_s5_tuned", "fa_s4_mfma", "fa_s3_fused", "fa_s5_combine", "fa_decode_split",
-                "fa_decode_combine"}
+    families = {"fa_s5_tuned", "fa_s5_parts", "fa_s4_mfma", "fa_s3_fused", "fa_s3_split",
+                "fa_s5_combine", "fa_decode_split", "fa_decode_combine"}
     seen = {fam for fam in families for name in kernels if fam in name}
     assert seen == families, f"missing from the report: {families - seen}"
     # Two dtypes x (12 D=64 + 8 D=128) stage-5 tiles.
     assert sum("fa_s5_tuned" in name for name in kernels) == 40
+
+
+def test_fp32_tiles_are_those_that_calls_reach(kernels):
+    """(D, RG, KS) of the fp32 kernel: what the tile rule picks, which includes the forced widths
+    (BC 32 and 64 at BR 128)."""
+    built = {tuple(int(x) for x in m.groups()) for name in kernels
+             if (m := re.search(r"fa_s3_splitILi(\d+)ELi(\d+)ELi(\d+)E", name))}
+    assert built == {(64, 4, 1), (64, 4, 2), (64, 2, 4), (64, 1, 4),
+                     (128, 4, 1), (128, 4, 2), (128, 2, 2)}
 
 
 # (dtype tag in the mangled name, D, RG, KS, BCW) -> occupancy (waves per SIMD) the launch
