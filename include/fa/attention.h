@@ -184,9 +184,9 @@ FA_API int fa_decode(int dtype, const void* q, const void* k, const void* v, voi
 
 /* Bytes of device scratch behind fa_decode_noalloc: one fixed array per GPU, held from the moment
  * the library's code is loaded on that GPU until the process ends. Sized for every problem the
- * automatic split count allows (num_splits = 0): that count keeps B*Hkv*S at most B*Hkv + 255
- * split groups at D = 128 and 512 at D = 64, and 510 groups of 64 rows of D = 128 fp32 partials
- * (plus their LSE) take 16,842,240 bytes. */
+ * automatic split count allows (num_splits = 0): where that count is not one, B*Hkv*S is at most
+ * 510 split groups at D = 128 and 512 at D = 64, and 510 groups of 64 rows of D = 128 fp32
+ * partials (plus their LSE) take 16,842,240 bytes. */
 #define FA_DECODE_SCRATCH_BYTES (17u << 20)
 
 /* fa_decode with no workspace argument and no allocation of any kind: the splits' partial O and

@@ -298,7 +298,7 @@ def test_noalloc_scratch_holds_every_automatic_split():
     """fa_decode_noalloc serves every problem whose split count the library picks itself
     (num_splits = 0): for B*Hkv from 1 to 300 split groups, up to 64 query rows per kv head and
     D = 64 or 128 on a long cache, the partials of the automatic split count fit the scratch
-    array. B*Hkv = 255 with 64 rows of D = 128 is the largest (2 splits, 16,842,240 bytes)."""
+    array. 510 split groups with 64 rows of D = 128 are the largest (16,842,240 bytes)."""
     lib = capi.load()
     text = HEADER.read_text()
     m = re.search(r"#define FA_DECODE_SCRATCH_BYTES \((\d+)u << (\d+)\)", text)
@@ -313,3 +313,26 @@ def test_noalloc_scratch_holds_every_automatic_split():
                 assert need <= capi.DECODE_SCRATCH_BYTES, (groups, g, nq, d, need)
                 worst = max(worst, need)
     assert worst == 16_842_240
+
+
+@pytest.mark.parametrize("d", [64, 128])
+def test_automatic_splits_keep_their_bounds(d):
+    """Over caches on both sides of every line of the split rule (short ones, four tiles per split, ten
+    tiles per CU, two rounds), up to 300 split groups and both workgroup heights: no split is empty or
+    shorter than a tile, splits never start a round that they do not fill, split groups stay within
+    the scratch array's 510 (D = 128) or 512 (D = 64), and a one-split call needs no workspace."""
+    lib = capi.load()
+    tiles_at = (list(range(1, 34)) + [37, 60, 95, 96, 97, 127, 128, 129, 255, 256, 257, 2047, 2048, 2049])
+    for groups in range(1, 301):
+        for tiles in sorted(set(tiles_at) | {max(1, (10 * 256 + e) // groups) for e in (-groups, -1, 0, groups)}):
+            for g, nq in ((1, 1), (64, 1)):
+                for nkv in (128 * (tiles - 1) + 1, 128 * tiles):
+                    p = capi.FaDecodeParams(groups, g, 1, nq, nkv, d, 0.125, True, 0)
+                    s = lib.fa_decode_num_splits(ctypes.byref(p))
+                    need = lib.fa_decode_workspace_bytes(capi.FA_DTYPE_F16, ctypes.byref(p))
+                    where = (groups, tiles, g, nq, d, s)
+                    assert 1 <= s <= tiles, where
+                    assert s == 1 or groups * s <= (512 if d == 64 else 510), where
+                    # One round of 256 (D = 64: 512) workgroups, or at D = 128 three halves of two.
+                    assert s == 1 or groups * s <= (512 if d == 64 else 256) or s == 3, where
+                    assert (need == 0) == (s == 1) and need <= capi.DECODE_SCRATCH_BYTES, where

@@ -6,8 +6,8 @@ more than one batch, contiguous operands and views of a packed projection. Every
 plain fp32 attention at the op's tolerance, O and LSE.
 
 Decode: the last cache that stays one split and the first that does not at each head dim and where half
-the CUs are busy, single-tile splits, the count where a split keeps four tiles, two
-workgroups per CU at D = 64, and one split per XCD there; each against the fp64 decode oracle.
+the CUs are busy, single-tile splits, the count where a split keeps four tiles, both sides of two
+workgroups per CU at D = 64 and of two rounds; each against the fp64 decode oracle.
 """
 
 from __future__ import annotations
@@ -51,12 +51,17 @@ def test_causal_walks_cut_by_length(b, h, hkv, n, d, dtype, monkeypatch):
 
 @pytest.mark.parametrize("b,hkv,group,nq,nkv,d", [
     (1, 8, 4, 1, 768, 128), (1, 8, 4, 1, 769, 128),     # one split, seven of a tile each
-    (4, 32, 1, 2, 896, 128), (4, 32, 1, 2, 897, 128),   # 128 groups: one, two
-    (3, 12, 2, 5, 896, 64), (3, 12, 2, 5, 897, 64),     # D = 64: one, seven
+    (4, 32, 1, 2, 896, 128), (4, 32, 1, 2, 897, 128),   # 128 groups: one
+    (4, 32, 1, 2, 1152, 128), (4, 32, 1, 2, 1153, 128), # and here one, two
+    (3, 12, 2, 5, 896, 64), (3, 12, 2, 5, 897, 64),     # D = 64: one
+    (3, 12, 2, 5, 1024, 64), (3, 12, 2, 5, 1025, 64),   # and here one, five
     (1, 1, 8, 1, 17000, 128),                           # 33 splits of four tiles and one more
     (8, 8, 4, 2, 8192, 64),                             # eight, two workgroups per CU
-    (3, 12, 2, 1, 4096, 64), (3, 12, 2, 1, 4632, 64),   # eight, one per XCD
-    (9, 8, 6, 8, 7680, 64),                             # seven, 8-wave workgroups
+    (3, 12, 2, 1, 4096, 64), (3, 12, 2, 1, 4632, 64),   # seven
+    (4, 10, 2, 1, 8064, 64), (4, 10, 2, 1, 8065, 64),   # 63 tiles: six, 64: twelve, two workgroups per CU
+    (10, 13, 1, 1, 6016, 128), (10, 13, 1, 1, 6017, 128),   # 130 groups: one, three in two rounds
+    (10, 17, 33, 1, 6017, 64),                          # 170, 8-wave workgroups: three
+    (9, 8, 6, 8, 7680, 64),                             # three, 8-wave workgroups
     (15, 17, 1, 1, 1100, 128),                          # 255 groups: one
 ], ids=lambda x: str(x))
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16], ids=["fp16", "bf16"])
@@ -65,7 +70,7 @@ def test_decode_automatic_splits(b, hkv, group, nq, nkv, d, dtype):
     q = _randn(gen, dtype, b, hkv * group, nq, d)
     k, v = (_randn(gen, dtype, b, hkv, nkv, d) for _ in range(2))
     o, lse = fused_attn.decode(q, k, v, is_causal=True)
-    ref, lse64 = decode_reference(q, k, v, is_causal=True)
     atol, rtol = O_TOL[dtype]
+    ref, lse64 = decode_reference(q, k, v, is_causal=True)
     assert_close_tol(o, ref, atol, rtol)
     assert_close_tol(lse.double().cpu().numpy(), lse64, LSE_ATOL, 0.0, what="LSE")
