@@ -8,7 +8,7 @@ For the attention kernels of the run (``fa_s*`` and ``fa_decode*``), per capture
 
 * duration: the mean kernel duration from the kernel trace (the last ``last`` dispatches when
   the program was bench.py's timed launches), TFLOP/s and share of the 2.5 PFLOP/s dense fp16/bf16
-  MFMA peak (157.3 TFLOP/s for fp32); split walks add the combine kernel's mean;
+  MFMA peak (a sixth of it for fp32, whose products are six bf16 ones); split walks add the combine kernel's mean;
 * launch: workgroups, waves per workgroup, VGPRs (architectural + accumulation), LDS bytes,
   scratch, and the occupancy they allow (waves per SIMD: 512 VGPRs per lane, 160 KiB of LDS per
   CU, at most one workgroup slot per 256 CUs per grid wave);
@@ -41,7 +41,7 @@ VGPRS_PER_LANE = 512      # unified architectural + accumulation file per SIMD l
 LDS_PER_CU = 160 * 1024
 MAX_WAVES_PER_SIMD = 8
 FETCH_SCALE, WRITE_SCALE = 2.0, 1.0
-PEAK = {"fp16": 2500.0, "bf16": 2500.0, "fp32": 157.3}  # dense MFMA TFLOP/s
+PEAK = {"fp16": 2500.0, "bf16": 2500.0, "fp32": 2500.0 / 6}  # dense MFMA TFLOP/s
 
 _TILE = re.compile(r"fa_s([45])_\w+?I(DF16_|DF16b)Li(\d+)ELi(\d+)ELi(\d+)ELi(\d+)E")
 
