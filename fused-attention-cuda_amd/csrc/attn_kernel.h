@@ -32,12 +32,14 @@
 // 32 lanes reading 32 different rows at the same column hit distinct banks (16 lanes x 16 B per
 // LDS cycle).
 //
-// Work distribution: grid = (N / BR) * B * H workgroups on a 1-D grid. Hardware hands workgroup i
-// to XCD (i + c) % 8, c fixed for the launch (8 XCDs, each with its own L2); the kernel remaps
-// blockIdx so that the workgroups of one residue i % 8 receive a contiguous range of
-// (head, q-tile) pairs, i.e. all Q tiles of a head sit on one XCD and its K/V is fetched into one
-// L2. For causal problems the heaviest Q tiles (longest key range) are issued
-// first within each XCD.
+// Work distribution: grid = (N / BR) * B * H workgroups on a 1-D grid, mapped by layout::grid_item as
+// in the 16-bit kernels. Hardware hands workgroup i to XCD (i + c) % 8, c fixed for the launch (8
+// XCDs, each with its own L2), so the workgroups of one residue i % 8 take a contiguous range of
+// (head, q-tile) pairs and a head's K/V is fetched into one L2. Causal grids issue the longest walks
+// first, of all heads of an XCD where it has whole ones: measured on MI355X, fp16, against head by
+// head, B8 H12 N1024 D64 209.5 -> 145.6 us, B16 H32 Hkv8 N512 D64 273 -> 172, B1 H16 N4096 D128 1082
+// -> 791. On other grids the order is the same as head by head (B2 H8 N2048 D64 162.9 and 163.6, B7
+// H7 N992 142.1 and 144.6).
 #pragma once
 
 #include <hip/hip_runtime.h>

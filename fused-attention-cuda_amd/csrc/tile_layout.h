@@ -201,13 +201,14 @@ FA_HD inline Item grid_item(int bid, int G, int n_qtiles, int splits, bool causa
 }
 
 // Causal split walks. Cutting every causal walk into the same number of parts leaves the parts as
-// unequal as the walks. Here a walk is cut by its length instead: with `unit` query tiles to a part,
-// query tile qt (its walk is qt + 1 query tiles' worth of keys) gets k = qt / unit + 1 parts, so no
-// part is longer than `unit` of them and most are near that. Tiles of one part need no merge and write
-// their output directly; the parts of the others have consecutive slots of BR partial rows in the
-// workspace, query tile by query tile: `base` is the first slot of qt. The launch ends with its longest
-// part: B1 H2 N8192 D128 bf16 75-78 us with two equal parts per walk (the longest 64 key tiles of
-// 64), 57-60 cut by length (43); B1 H1 N8192 65 and 50, B2 H1 N2048 D128 fp16 19.1 and 17.4.
+// unequal as the walks. Here a walk is cut by its length instead: with `unit` query tiles to a
+// part, query tile qt (its walk is qt + 1 query tiles' worth of keys) gets k = qt / unit + 1 parts,
+// so no part is longer than `unit` of them and most are near that. Tiles of one part need no merge
+// and write their output directly; the parts of the others have consecutive slots of BR partial
+// rows in the workspace, query tile by query tile: `base` is the first slot of qt. The launch ends
+// with its longest part: B1 H2 N8192 D128 bf16 75-78 us with two equal parts per walk (the longest
+// 64 key tiles of 64), 57-60 cut by length (43); B1 H1 N8192 65 and 50, B2 H1 N2048 D128 fp16 19.1
+// and 17.4.
 FA_HD constexpr int parts_base(int unit, int qt, int k) {
   return k < 2 ? 0 : unit * ((k - 1) * k / 2 - 1) + (qt - (k - 1) * unit) * k;
 }
@@ -223,8 +224,8 @@ struct PartItem {
   int part;
   int k;
 };
-// Work item idx of a head, most parts per tile first (their tiles have the longest walks). div_k(x, k)
-// must return x / k.
+// Work item idx of a head, most parts per tile first (their tiles have the longest walks). div_k(x,
+// k) must return x / k.
 template <typename DivK>
 FA_HD inline PartItem parts_item(int idx, int unit, int n_qtiles, DivK div_k) {
   int k = (n_qtiles - 1) / unit + 1;
@@ -250,7 +251,8 @@ FA_HD inline PartItem parts_item(int idx, int unit, int n_qtiles, DivK div_k) {
 FA_HD inline int parts_unit(int n_qtiles, int br, int N, int splits, long long heads,
                             long long resident, int max_parts) {
   const int longest = (n_qtiles + splits - 1) / splits;
-  // Parts of fewer than 256 keys are mostly fixed cost (B1 H1 N1024 D128: 11.9 us with parts of 64).
+  // Parts of fewer than 256 keys are mostly fixed cost (B1 H1 N1024 D128: 11.9 us with parts of
+  // 64).
   const int fewest = 256 / br > 1 ? 256 / br : 1;
   const int least = (n_qtiles + max_parts - 1) / max_parts;
   for (int unit = least > fewest ? least : fewest; unit < longest; ++unit) {

@@ -317,14 +317,16 @@ def test_noalloc_scratch_holds_every_automatic_split():
 
 @pytest.mark.parametrize("d", [64, 128])
 def test_automatic_splits_keep_their_bounds(d):
-    """Over caches on both sides of every line of the split rule (short ones, four tiles per split, ten
-    tiles per CU, two rounds), up to 300 split groups and both workgroup heights: no split is empty or
-    shorter than a tile, splits never start a round that they do not fill, split groups stay within
-    the scratch array's 510 (D = 128) or 512 (D = 64), and a one-split call needs no workspace."""
+    """Over caches on both sides of every line of the split rule (short ones, four tiles per split,
+    ten tiles per CU, two rounds), up to 300 split groups and both workgroup heights: no split is
+    empty or shorter than a tile, splits never start a round that they do not fill, split groups stay
+    within the scratch array's 510 (D = 128) or 512 (D = 64), and a one-split call needs no
+    workspace."""
     lib = capi.load()
-    tiles_at = (list(range(1, 34)) + [37, 60, 95, 96, 97, 127, 128, 129, 255, 256, 257, 2047, 2048, 2049])
+    lines = {*range(1, 34), 47, 48, 49, 60, 127, 128, 129, 256, 2048, 2049}
     for groups in range(1, 301):
-        for tiles in sorted(set(tiles_at) | {max(1, (10 * 256 + e) // groups) for e in (-groups, -1, 0, groups)}):
+        ten_per_cu = {max(1, (10 * 256 + e) // groups) for e in (-groups, -1, 0, groups)}
+        for tiles in sorted(lines | ten_per_cu):
             for g, nq in ((1, 1), (64, 1)):
                 for nkv in (128 * (tiles - 1) + 1, 128 * tiles):
                     p = capi.FaDecodeParams(groups, g, 1, nq, nkv, d, 0.125, True, 0)

@@ -1,9 +1,9 @@
 """fp32 forward on split bf16 operands (stage 3, ``fa_s3_split``) against the fp64 oracle.
 
-Sizes: both sides of every tile edge (32-row workgroups up to 128-row ones, partial last tiles of 32,
-64 and 128 keys), each tile the rule can pick, GQA, strided views. Values: very different magnitudes side
-by side, and everything that must leave the split path for the fp32 matrix instructions (magnitudes
-from 2^60 on, nonzero ones below 2^-110, infinities).
+Sizes: both sides of every tile edge (32-row workgroups up to 128-row ones, partial last tiles of
+32, 64 and 128 keys), each tile the rule can pick, GQA, strided views. Values: very different
+magnitudes side by side, and everything that must leave the split path for the fp32 matrix
+instructions (magnitudes from 2^60 on, nonzero ones below 2^-110, infinities).
 
 The bar is the fp32 one of the other parity tests (|O err| <= 1e-5 + 1e-5 |ref|). With scaled V the
 absolute part scales with V: every term of the error is proportional to it.
@@ -44,8 +44,8 @@ def _check(q, k, v, causal, v_scale=1.0, atol=1e-5):
     (1, 1, 1, 32, 64), (1, 2, 1, 96, 64), (1, 2, 2, 160, 64),       # BR 32 x BC 128
     (1, 2, 2, 32, 128), (1, 2, 1, 96, 128), (1, 2, 2, 352, 128),    # BR 64 x BC 64
     (3, 16, 4, 288, 64),                                            # BR 64 x BC 128
-    (4, 16, 4, 288, 64), (4, 16, 8, 288, 128),                      # BR 128 x BC 64 (causal 64 rows)
-    (4, 24, 8, 352, 64),                                            # causal longer than its grid's rounds
+    (4, 16, 4, 288, 64), (4, 16, 8, 288, 128),              # BR 128 x BC 64 (causal 64 rows)
+    (4, 24, 8, 352, 64),                                    # BR 64 x BC 128 in three rounds
     (2, 2, 1, 32, 128), (9, 32, 8, 96, 128),                        # one narrow tile per head
     (8, 32, 8, 352, 64), (8, 32, 8, 288, 128),                      # BR 128 x BC 32
 ], ids=lambda s: "B%d_H%d_Hkv%d_N%d_D%d" % s)
@@ -64,8 +64,8 @@ def test_forced_widths(d, bc):
         fused_attn.set_debug_overrides(0, 0)
 
 
-# Largest magnitude of a tensor at ordinary sizes, at the upper end of the split path's range, 2^60, and
-# past it. q and k scale against each other, so that the scores keep the size of ordinary ones.
+# Largest magnitude of a tensor at ordinary sizes, at the upper end of the split path's range, 2^60,
+# and past it. q and k scale against each other, so that the scores keep the size of ordinary ones.
 @pytest.mark.parametrize("top", [2.0 ** -7, 2.0 ** -6, 0.5, 2.0 ** 9 - 2.0 ** -14, 2.0 ** 9,
                                  2.0 ** 60 - 2.0 ** 36, 2.0 ** 60, 1e30], ids=lambda x: "%g" % x)
 @pytest.mark.parametrize("which", ["q", "k", "v"])
@@ -88,12 +88,12 @@ def test_range_ends(which, top):
 @pytest.mark.parametrize("d", [64, 128])
 @pytest.mark.parametrize("tensor", [0, 1, 2], ids=["q", "k", "v"])
 def test_one_row_of_another_size(tensor, d, factor):
-    """One row of the last tile far larger than the rest, or outside the range, whose workgroups start over
-    on the fp32 path after tiles of the split one. Everything that the row does not decide keeps the
-    ordinary bar; the terms it has a part in add what fp32 leaves of them."""
+    """One row of the last tile far larger than the rest, or outside the range, whose workgroups start
+    over on the fp32 path after tiles of the split one. Everything that the row does not decide keeps
+    the ordinary bar; the terms it has a part in add what fp32 leaves of them."""
     x = list(_inputs(1, 2, 2, 416, d, seed=3))
     x[tensor][0, 0, 401] *= factor
-    if factor > 1e18 and tensor < 2:  # scores of ordinary size for the row, next to nothing for the others
+    if factor > 1e18 and tensor < 2:  # scores of ordinary size for the row, none for the others
         x[1 - tensor] /= factor
     q, k, v = x
     o, _ = fused_attn.forward_stage(q, k, v, 3)
@@ -102,11 +102,11 @@ def test_one_row_of_another_size(tensor, d, factor):
     qd, kd, vd = (t[0, 0].double() for t in x)
     p = torch.softmax(qd @ kd.t().contiguous() / math.sqrt(d), dim=-1)
     if tensor == 2:
-        # A sum of 416 products, each weight off by a few ulp of a score of size 4: 1e-6 of the terms.
+        # A sum of 416 products, each weight off by a few ulp of a score of size 4: 1e-6 of them.
         bar[0, 0] += 1e-6 * (p @ vd.abs()).cpu().numpy()
     elif factor == 2e3:
-        # A score of D products is off by at most D 2^-24 of their magnitudes; it moves O by p (1 - p) of
-        # that, times the spread of v.
+        # A score of D products is off by at most D 2^-24 of their magnitudes; it moves O by
+        # p (1 - p) of that, times the spread of v.
         s_err = d * 2.0 ** -24 * (qd.abs() @ kd.abs().t().contiguous()) / math.sqrt(d)
         move = (s_err * p * (1 - p)).sum(dim=-1, keepdim=True) * 2 * vd.abs().max()
         bar[0, 0] += move.cpu().numpy()
@@ -176,8 +176,9 @@ def _column_errors(o, ref):
     return err.max(axis=(0, 1, 2)) / np.abs(ref).max(axis=(0, 1, 2))
 
 
-# Values of very different magnitude side by side: an fp32 product keeps 24 bits of each operand whatever
-# stands beside it, so every output is held to its own magnitude. The bar is the fp32 one, 1e-5 of it.
+# Values of very different magnitude side by side: an fp32 product keeps 24 bits of each operand
+# whatever stands beside it, so every output is held to its own magnitude. The bar is the fp32 one,
+# 1e-5 of it.
 @pytest.mark.parametrize("small", [1e-3, 1e-6, 1e-10, 1e-25, 1e-36], ids=lambda x: "%g" % x)
 @pytest.mark.parametrize("d", [64, 128])
 def test_small_v_columns_beside_large_ones(d, small):
